@@ -3480,7 +3480,8 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
 // in piece order and dE is written in the pass's mode, as the sums' epilogue writes a
 // whole task.  32 workgroups per task, 4 of its rows each; a thread takes 4 columns of
 // one row and adds the npc pieces' values with four sums in flight.  The grid covers
-// the most tasks that can be cut (at most kDePartSlots / 2: two pieces each at least).
+// the most tasks that can be cut (de_cut_tasks_max), whatever part of the token blocks
+// keeps tiles; workgroups past the cut tasks end at once.
 constexpr int kDePiecesPerTask = kBwdTokens / 4;
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_de_pieces_kernel(BwdArgs a, int chunk, int pass, int nwg) {
@@ -3737,17 +3738,15 @@ static hipError_t backward_typed(const BwdArgs& a, hipStream_t s, hipEvent_t pas
         launch_sum<T, 0>(ac, wide_de, chunk, pass, gp, s);
         if ((e2 = hipGetLastError()) != hipSuccess) return e2;
         if (!wide_de && a.de_part != nullptr) {  // pieces of dE tasks (de_pieces_of)
-          if (P.nrb * ((a.D + kDePartCols - 1) / kDePartCols) > gp) {  // tasks may overflow the grid
+          const int64_t tasks = P.nrb * ((a.D + kDePartCols - 1) / kDePartCols);
+          if (tasks > gp) {  // tasks may overflow the grid
             BwdArgs a1 = ac;
             a1.de_stage = 1;
             launch_sum<T, 0>(a1, false, chunk, pass, gp, s);
             if ((e2 = hipGetLastError()) != hipSuccess) return e2;
           }
-          // no more tasks can be cut than there are, nor than leave two pieces each
-          const int64_t tasks = P.nrb * ((a.D + kDePartCols - 1) / kDePartCols);
-          const int64_t ncut = tasks > gp ? tasks - gp : tasks;
-          const unsigned pg = (unsigned)(kDePiecesPerTask * (ncut < kDePartSlots / 2 ? ncut : kDePartSlots / 2));
-          hipLaunchKernelGGL((bwd_de_pieces_kernel<T>), dim3(pg), dim3(256), 0, s, a, chunk, pass, gp);
+          hipLaunchKernelGGL((bwd_de_pieces_kernel<T>), dim3((unsigned)(kDePiecesPerTask * de_cut_tasks_max(tasks, gp))),
+                             dim3(256), 0, s, a, chunk, pass, gp);
           if ((e2 = hipGetLastError()) != hipSuccess) return e2;
         }
       }

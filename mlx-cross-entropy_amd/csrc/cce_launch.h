@@ -152,6 +152,13 @@ enum WriteMode { kWriteT = 0, kStoreF32 = 1, kAddF32 = 2, kFinishT = 3, kPartF32
 // pieces of the tasks past the grid.
 constexpr int kDePartSlots = 256;  // pieces at most (fp32 slots of 128 x 256 sums)
 constexpr int kDePartCols = 256;   // the narrow sums' D slice
+// The most tasks a pass can cut on a grid of nwg workgroups, given the most tasks it can have:
+// the host does not know how many token blocks keep tiles in the pass, and few of many leave
+// as many cut tasks as few of few (two pieces each at least).
+inline int64_t de_cut_tasks_max(int64_t tasks, int nwg) {
+  const int64_t most = (nwg < kDePartSlots ? nwg : kDePartSlots) / 2;
+  return tasks < most ? tasks : most;
+}
 
 struct BwdPlan {
   int64_t nvt, nrb, total;  // vocab tiles, token blocks, pairs

@@ -441,7 +441,12 @@ def test_g_tile_tasks_cover_every_kept_pair_once(seed):
 
 DE_PART_SLOTS = 256  # kDePartSlots: fp32 partial sums of 128 x 256 outputs each
 DE_PIECES_PER_TASK = 128 // 4  # kDePiecesPerTask: 4 of a task's 128 rows per workgroup
-DE_PIECES_GRID = DE_PIECES_PER_TASK * (DE_PART_SLOTS // 2)  # kDePiecesGrid: bwd_de_pieces_kernel
+
+
+def de_pieces_grid(nrb, nds, nwg):
+    """bwd_de_pieces_kernel's workgroups: the host knows the plan's most tasks (every token
+    block x the D slices), not how many blocks keep tiles in the pass (de_cut_tasks_max)."""
+    return DE_PIECES_PER_TASK * min(nrb * nds, min(nwg, DE_PART_SLOTS) // 2)
 
 
 def de_pieces_of(ntasks, nwg):
@@ -507,6 +512,7 @@ def test_de_pieces_cover_every_task_tile_once(seed):
     nown = int(rng.choice([1, 2, 3, 4, 8, 16, 32, 64, 65, 128, 288, 300, 384, 400]))
     nds = int(rng.choice([1, 1, 2, 9, 16]))
     nwg = int(rng.choice([8, 200, 256, 304]))
+    nrb = nown + int(rng.choice([0, 0, 1, 9, 100]))  # token blocks, the others without kept tiles
     own_cnt = [int(x) for x in rng.integers(1, 400, nown)]
     own_cnt[-1] = int(rng.choice([1, 2, own_cnt[-1]]))  # owners with fewer tiles than pieces
     npc, pieces, whole, fin = de_pieces_restated(own_cnt, nds, nwg)
@@ -531,11 +537,23 @@ def test_de_pieces_cover_every_task_tile_once(seed):
         assert sorted(sum(fin.values(), [])) == sorted(pieces)
         # its workgroups (cut task index = block // 32, rows 4 (block % 32) + wave) reach
         # every row of every cut task
-        rows = {(b // DE_PIECES_PER_TASK, 4 * (b % DE_PIECES_PER_TASK) + w) for b in range(DE_PIECES_GRID) for w in range(4)}
+        grid = de_pieces_grid(nrb, nds, nwg)
+        rows = {(b // DE_PIECES_PER_TASK, 4 * (b % DE_PIECES_PER_TASK) + w) for b in range(grid) for w in range(4)}
         assert rows >= {(ti, m) for ti in range(ncut) for m in range(128)}
     # each workgroup runs at most one item per launch when anything is cut
     if npc > 1:
         assert len({v for v, _ in whole}) == len(whole)
+
+
+@pytest.mark.parametrize("nwg", [8, 104, 200, 256, 304])
+@pytest.mark.parametrize("nds", [1, 2, 3, 9, 16, 32])
+def test_de_pieces_grid_covers_any_live_blocks(nds, nwg):
+    """Whatever part of the token blocks keeps tiles in a pass (masked rows, a late pass or
+    chunk), the finisher has workgroups for every task that the sums cut."""
+    for nrb in range(1, 3 * DE_PART_SLOTS // 2 // nds + 1):
+        reach = de_pieces_grid(nrb, nds, nwg) // DE_PIECES_PER_TASK
+        for nown in range(nrb + 1):
+            assert de_pieces_of(nown * nds, nwg)[1] <= reach, (nrb, nown)
 
 
 def test_de_pieces_mutant_is_caught():

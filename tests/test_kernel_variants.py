@@ -360,3 +360,30 @@ def test_loss_of_confident_rows(m, cuda, layout_ref):
     nll = m._ext.forward(e, c, t, ref_stats=layout_ref)[4]
     want = torch.log1p((V - 1) * torch.exp(-e[:, 0].double()))
     assert ((nll.double() - want).abs() <= 2e-5 * want + 2.0 ** -18).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", [dict(), dict(max_g_tiles=1), dict(max_chunk_tiles=32)])
+@pytest.mark.parametrize("order", ["input", "sorted"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,D,masked", [(2176, 4096, 1152), (4096, 2304, 2304), (2176, 4096, 2000)])
+def test_de_pieces_of_masked_token_blocks(m, cuda, N, D, masked, dtype, order, split):
+    """More than 256 dE tasks by the sizes, but over half of the token blocks hold only ignored rows:
+    the tasks that are left are cut into pieces, and every one of them is finished (dE starts from
+    memory that holds NaN).  Against whole tasks: fp32 sums in another order (1e-5), 16-bit outputs
+    rounded from them (2e-3), as without masked rows."""
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the task counts are laid out for a 256-workgroup grid")
+    e, c, t = _case(N, D, 9000, dtype, cuda, seed=37, std=0.05)
+    t[N - masked:] = -100
+    tm, _, _, lse, _ = m._ext.forward(e, c, t)
+    d = torch.linspace(0.5, 1.5, N, device=cuda)
+    out = []
+    for tasks in (None, "whole"):
+        used = torch.full_like(e, float("nan"))  # the next tensor of this size takes its memory
+        del used
+        with m._ext.backward_options(token_order=order, de_tasks=tasks, **split):
+            out.append(m._ext.backward(e, c, t, lse, tm, d, want_dc=False)[0])
+    assert torch.isfinite(out[0]).all()
+    err = (out[0].double() - out[1].double()).norm() / out[1].double().norm()
+    assert err <= (1e-5 if dtype == torch.float32 else 2e-3)
