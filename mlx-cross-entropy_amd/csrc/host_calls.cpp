@@ -97,8 +97,12 @@ struct Operands {
   }
 };
 
+// What the general path passes for o: int(o), its low 64 bits (ctypes' conversion).
 bool int_of(PyObject* o, int64_t& v) {
-  v = PyLong_AsLongLong(o);
+  PyObject* i = PyNumber_Long(o);
+  if (!i) return false;
+  v = (int64_t)PyLong_AsUnsignedLongLongMask(i);
+  Py_DECREF(i);
   return !(v == -1 && PyErr_Occurred());
 }
 

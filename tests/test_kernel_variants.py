@@ -1,6 +1,7 @@
 """Variants a dispatch chooses by size, type or layout, at the sizes where each can go wrong,
 against the path they stand in for or the float64 oracle."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -245,6 +246,23 @@ def test_native_host_calls_match_the_general_path(m, cuda, dtype, reduction):
     for other in out[1:]:
         for x, y in zip(out[0], other):
             assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ignore", [-100.0, np.float32(-100), np.int32(-100), torch.tensor(-100), "-100", 2 ** 64 - 100])
+def test_native_host_calls_take_any_ignore_index(m, cuda, ignore):
+    """ignore_index goes through int() whatever the operands' layout: the native call and the general
+    path (int32 targets) take the same values, and refuse the same."""
+    e, c, t = _case(60, 24, 300, torch.bfloat16, cuda, seed=4)
+    t[::4] = -100
+    want = m.linear_cross_entropy(e, c, t)
+    for tt in (t, t.to(torch.int32)):
+        x = e.detach().requires_grad_()
+        loss = m.linear_cross_entropy(x, c, tt, ignore_index=ignore)
+        dE, = torch.autograd.grad(loss, x)
+        assert torch.equal(loss, want) and (dE[::4] == 0).all()
+        with pytest.raises(ValueError):
+            m.linear_cross_entropy(e, c, tt, ignore_index="none")
 
 
 @pytest.mark.gpu
