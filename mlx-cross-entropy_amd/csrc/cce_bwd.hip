@@ -3305,7 +3305,11 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
                     (PHASE == 0 ? c.h * (S::KS * 4) : c.h * (S::KS * kBwdVocab * 4));
     gr = gld16(g + goff);
   };
-  float mx = 0.f;
+  float mx = 0.f;  // the largest magnitude of the task's operands
+  auto max4 = [&](const u32x4& r) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mx = fmaxf(mx, fabsf(__uint_as_float(r[k])));
+  };
   auto cut4 = [&](const u32x4& r, char* at, int plane) {
     uint32_t p[3][2];
 #pragma unroll
@@ -3465,10 +3469,19 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
       cs.h = 0;
       if (++cs.j == cs.cnt) break;
     }
-    // (mx also covers the next task's first step: at worst a task is computed twice)
+    // (mx also covers the next task's first step, stored already: at worst the task before
+    // one that has to be is computed twice)
     if (mx > kBf16Max) *flag = 1;
     stage_barrier<63>();
-    if (__builtin_expect(*flag != 0, 0)) redo(cs);
+    if (__builtin_expect(*flag != 0, 0)) {
+      redo(cs);
+      __syncthreads();                  // every wave has read the flag
+      if (threadIdx.x == 0) *flag = 0;  // (set again a whole task of barriers from here at the earliest)
+    }
+    mx = 0.f;  // the next task's, from its first step (still in registers)
+    max4(xr[0]);
+    max4(xr[1]);
+    max4(gr);
     epilogue(cs);
     if (!seek(cs.q + 1, cs)) break;
   }

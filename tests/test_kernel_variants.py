@@ -223,6 +223,31 @@ def test_fp32_infinite_operands(m, cuda, N, D, V, filter_eps):
 
 
 @pytest.mark.gpu
+def test_fp32_infinite_operand_stays_with_its_tasks(m, cuda):
+    """An infinite classifier entry has the dE tasks of its 256 columns computed on the fp32 path, and not
+    later tasks of the same workgroup: 600 tasks on 256 workgroups here, where a third of them take a
+    task of the last 256 columns after one of the first.  The last columns are the same bits as with a
+    finite entry of the same effect.  (Whole-number operands: exact logits either way, so G is the
+    same; dE's sums depend on the path in their last bits.)"""
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the tasks are laid out for a 256-workgroup grid")
+    N, D, V = 200 * 128, 768, 256
+    g = torch.Generator(device=cuda).manual_seed(5)
+    e = torch.randint(-1, 2, (N, D), generator=g, device=cuda).float()
+    c = torch.randint(-8, 9, (V, D), generator=g, device=cuda).float() / 64
+    e[:, 0] = 1.0
+    t = torch.randint(8, V, (N,), generator=g, device=cuda)
+    out = []
+    for entry in (-1e4, -float("inf")):
+        c[7, 0] = entry
+        tm, _, _, lse, _ = m._ext.forward(e, c, t)
+        dE = m._ext.backward(e, c, t, lse, tm, torch.ones(N, device=cuda), filter_eps=None, want_dc=False)[0]
+        out.append((lse, dE[:, 512:]))
+    assert torch.equal(out[0][0], out[1][0])
+    assert torch.isfinite(out[0][1]).all() and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("reduction", ["none", "sum", "mean"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_native_host_calls_match_the_general_path(m, cuda, dtype, reduction):
