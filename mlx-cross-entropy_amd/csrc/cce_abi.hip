@@ -399,7 +399,7 @@ int backward_impl(int dtype, const void* e, const void* c, const void* bias, con
   a.tile_stats = tile_stats;
   a.dc_zeroed = (flags & CCE_BWD_DC_ZEROED) ? 1 : 0;
   a.stats32 = (flags & CCE_BWD_REF_STATS) ? 1 : 0;
-  a.g_scaled = dtype == CCE_DTYPE_F16 ? 1 : 0;  // fp16 G tiles are scaled into fp16's normal range
+  a.g_scaled = dtype != CCE_DTYPE_BF16 ? 1 : 0;  // G tiles scaled into fp16's normal range, in fp32 into the cut's
   a.g_split = P.g_split ? 1 : 0;  // the layout the plan's slots are sized for
   // one-tile dC owners by token block: 16-bit inputs with G rounded once
   a.dc_blk = es == 2 && !a.g_split && dC != nullptr && P.nrb <= cce::kDcBlkMaxRb && !(flags & CCE_BWD_DC_OWNER_TASKS);

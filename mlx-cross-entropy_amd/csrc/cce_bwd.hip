@@ -700,11 +700,41 @@ __device__ __forceinline__ int order_by_size(int n, F size, int* out, int base, 
 constexpr int kGPairRounds = 2;  // pair tasks up to this many per workgroup
 constexpr int kRbsLds = 8192;  // (pass, token block) slot starts held in LDS when they fit
 
+// The scale of the G tiles (counts[kGScaleExp]), by one workgroup of 1024 threads.
+// fp16: s with max |d_nll| 2^s in [2^13, 2^14) (|G| <= |d_nll|), so G * 2^s neither
+// overflows fp16 nor meets its subnormals above 2^-10 of the largest value.  fp32: in
+// [2^50, 2^51), so that what the sums' cut loses (2^-134 of a value) is nothing beside even a row
+// of G that is all near 2^-126 of the largest value.  0 when every d_nll is 0 or one is not finite.
+__device__ __forceinline__ void g_scale(const BwdArgs& a, uint32_t* wmax) {
+  const int tid = threadIdx.x;
+  uint32_t mb = 0u;
+  for (int64_t r = tid; r < a.N; r += 1024) mb = max(mb, __float_as_uint(a.d_nll[r]) & 0x7fffffffu);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
+  if ((tid & 63) == 0) wmax[tid >> 6] = mb;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < 16; ++w) mb = max(mb, wmax[w]);
+    const int top = a.plan.esize == 4 ? 51 : 14;
+    int se = 0;
+    if (mb >= 0x7f800000u || mb == 0u) se = 0;
+    else if (mb < 0x00800000u) se = 120;  // subnormal
+    else se = min(120, top - ((int)(mb >> 23) - 126));
+    a.counts[kGScaleExp] = se;
+  }
+}
+
 __global__ __launch_bounds__(1024) void bwd_compact_kernel(BwdArgs a, int chunk) {
   // Workgroups past the first copy the rows into the sorted order (16 rows each, one
   // per wave) while the first compacts: the copy does not wait for the choice of
-  // order, and is only read if the sorted order is chosen.
+  // order, and is only read if the sorted order is chosen.  With a.g_scaled the first chunk's
+  // last workgroup finds the G tiles' scale.
   if (blockIdx.x > 0) {
+    if (a.g_scaled && chunk == 0 && blockIdx.x + 1 == gridDim.x) {
+      __shared__ uint32_t wmax[16];
+      g_scale(a, wmax);
+      return;
+    }
     permute_row(a, (int64_t)(blockIdx.x - 1) * 16 + (threadIdx.x >> 6), a.D * (int64_t)a.plan.esize);
     return;
   }
@@ -757,27 +787,6 @@ __global__ __launch_bounds__(1024) void bwd_compact_kernel(BwdArgs a, int chunk)
   }
   __syncthreads();
   const uint32_t* bsrc = sorted ? a.bits_p : a.bits;
-  if (chunk == 0 && a.g_scaled) {
-    // fp16 G tiles: s with max |d_nll| 2^s in [2^13, 2^14) (|G| <= |d_nll|), so G * 2^s
-    // neither overflows fp16 nor meets its subnormals above 2^-10 of the largest
-    // value; 0 when every d_nll is 0 or one is not finite.
-    uint32_t mb = 0u;
-    for (int64_t r = tid; r < a.N; r += 1024) mb = max(mb, __float_as_uint(a.d_nll[r]) & 0x7fffffffu);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
-    if ((tid & 63) == 0) wsum[tid >> 6] = (int)mb;
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 1; w < 16; ++w) mb = max(mb, (uint32_t)wsum[w]);
-      int se = 0;
-      if (mb >= 0x7f800000u || mb == 0u) se = 0;
-      else if (mb < 0x00800000u) se = 120;  // subnormal
-      else se = min(120, 14 - ((int)(mb >> 23) - 126));
-      a.counts[kGScaleExp] = se;
-    }
-    __syncthreads();
-  }
-
   for (int e = tid; e < E; e += 1024) {
     const int rb = e / cwd, wl = e - rb * cwd;
     uint32_t x = bsrc[(size_t)rb * nw + wlo + wl];
@@ -1493,7 +1502,7 @@ constexpr int kGThreads = GLoop<__bf16>::NTHREADS;
 // of vocabulary v0 + 32 i + 8 (r/4) + 4 h + r%4 and token tok0 + 32 j + n.  Stored
 // token-major into the slot's G tile gtile at rows row0 + 32 j + n: fp32 as it is,
 // 16-bit types rounded once (rows of 128 columns) or, with a.g_split, as the hi / lo
-// pair of g_tile_bytes's layout (fp16 scaled by 2^gexp either way); with WANT_DB the
+// pair of g_tile_bytes's layout (fp16 and fp32 scaled by 2^gexp); with WANT_DB the
 // block's (unscaled) column sums over its 64 tokens go to red[0, 128).  Per token: g (0 for masked / out-of-range rows), lz =
 // lse log2(e), or +inf when g == 0 so that p = 0 and G = 0 without a select, and the
 // target's place in the block as tl - 4 h, which register (i, r) holds iff it equals
@@ -1521,7 +1530,7 @@ __device__ __forceinline__ GRows g_rows_load(const BwdArgs& a, const RowData& rd
   return r;
 }
 
-// The exponent s of the fp16 G tiles' scale 2^s (0 unless a.g_scaled).
+// The exponent s of the fp16 and fp32 G tiles' scale 2^s (0 unless a.g_scaled).
 __device__ __forceinline__ int g_scale_exp(const BwdArgs& a) { return a.g_scaled ? ldu(a.counts, kGScaleExp) : 0; }
 
 template <typename T, bool HAS_BIAS, bool WANT_G, bool WANT_DB, int TI = 4>
@@ -1532,9 +1541,9 @@ __device__ __forceinline__ void g_block_epilogue(const BwdArgs& a, const RowData
   const int lane = threadIdx.x & 63;
   const int n = lane & 31, h = lane >> 5;
   const T* bias = reinterpret_cast<const T*>(a.bias);
-  // fp16: G is formed as (d_nll 2^s) (p - onehot), exact scaling by a power of two;
+  // fp16, fp32: G is formed as (d_nll 2^s) (p - onehot), exact scaling by a power of two;
   // the column sums take it back out
-  const int gexp = ES == 2 ? g_scale_exp(a) : 0;
+  const int gexp = g_scale_exp(a);
   const float gmul = __builtin_ldexpf(1.f, gexp), gdiv = __builtin_ldexpf(1.f, -gexp);
   float g[TJ], lz[TJ];
   int tl[TJ];
@@ -1657,7 +1666,7 @@ __device__ __forceinline__ void g_block_epilogue(const BwdArgs& a, const RowData
         sm += __shfl_xor(sm, 4);
         sm += __shfl_xor(sm, 8);
         sm += __shfl_xor(sm, 16);
-        if (n == 0) red[i * 32 + (r >> 2) * 8 + h * 4 + (r & 3)] = ES == 2 ? sm * gdiv : sm;
+        if (n == 0) red[i * 32 + (r >> 2) * 8 + h * 4 + (r & 3)] = sm * gdiv;
       }
     }
   }
@@ -3305,17 +3314,20 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
                     (PHASE == 0 ? c.h * (S::KS * 4) : c.h * (S::KS * kBwdVocab * 4));
     gr = gld16(g + goff);
   };
-  float mx = 0.f;  // the largest magnitude of the task's operands
-  auto max4 = [&](const u32x4& r) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) mx = fmaxf(mx, fabsf(__uint_as_float(r[k])));
+  // The range of the task's operands.  Products and sums of operands up to 2^52 stay finite (G is
+  // scaled to at most 2^51); larger ones, and others the cut is not for (NTMainLoop<float>), take redo.
+  constexpr float kTop = 4503599627370496.f;
+  CutRange<3> range;  // of the X rows wave and wave + 8 of the steps, and of G
+  auto see4 = [&](int j, const u32x4& r) {
+    range.see(j, __uint_as_float(r[0]), __uint_as_float(r[1]));
+    range.see(j, __uint_as_float(r[2]), __uint_as_float(r[3]));
   };
-  auto cut4 = [&](const u32x4& r, char* at, int plane) {
+  auto cut4 = [&](int j, const u32x4& r, char* at, int plane) {
     uint32_t p[3][2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       float x0 = __uint_as_float(r[2 * k]), x1 = __uint_as_float(r[2 * k + 1]);
-      mx = fmaxf(mx, fmaxf(fabsf(x0), fabsf(x1)));
+      range.see(j, x0, x1);
 #pragma unroll
       for (int t = 0; t < 3; ++t) {
         p[t][k] = cvt_bf16x2(x0, x1);
@@ -3328,7 +3340,8 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
   };
 
   f32x16 acc[2][2];
-  // The task once more on fp32 MFMAs, fragments from memory (an operand was infinite).
+  const float gdiv = __builtin_ldexpf(1.f, -g_scale_exp(a));  // G tiles hold G 2^gexp: scaled back (exact)
+  // The task once more on fp32 MFMAs, fragments from memory, G unscaled.
   auto redo = [&](Cur c) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -3350,7 +3363,7 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
 #pragma unroll
           for (int jj = 0; jj < 2; ++jj) {
             const int m = wm * 64 + 32 * jj + n;
-            gf[jj][q] = __float_as_uint(PHASE == 0 ? G[m * kBwdVocab + k0 + q] : G[(k0 + q) * kBwdVocab + m]);
+            gf[jj][q] = __float_as_uint((PHASE == 0 ? G[m * kBwdVocab + k0 + q] : G[(k0 + q) * kBwdVocab + m]) * gdiv);
           }
         }
 #pragma unroll
@@ -3360,8 +3373,8 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
       }
     }
   };
-  // acc[i][jj][r]: output column ds DN + 64 wd + 32 i + 8 (r/4) + 4 h + r%4 of row 64 wm + 32 jj + n.
-  auto epilogue = [&](const Cur& c) {
+  // acc[i][jj][r] * unscale: output column ds DN + 64 wd + 32 i + 8 (r/4) + 4 h + r%4 of row 64 wm + 32 jj + n.
+  auto epilogue = [&](const Cur& c, float unscale) {
     const int64_t orow0 = (int64_t)(PHASE == 0 ? c.owner : vlo + c.owner) * 128;
     const int64_t orows = PHASE == 0 ? a.N : a.V;
     const int64_t nrows = orows - orow0 < 128 ? orows - orow0 : 128;
@@ -3383,6 +3396,7 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
           const int64_t d = (int64_t)c.ds * S::DN + wd * 64 + 32 * i + 8 * q + 4 * h;
           if (d >= D) continue;
           f32x4 v{acc[i][jj][4 * q], acc[i][jj][4 * q + 1], acc[i][jj][4 * q + 2], acc[i][jj][4 * q + 3]};
+          v *= unscale;
           f32x4* cp = reinterpret_cast<f32x4*>(carry + m * cstride + d);
           if (mode == kWriteT) {
             *reinterpret_cast<f32x4*>(orow + d) = v;
@@ -3408,8 +3422,8 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
   auto stash = [&](int st) {
     char* sp = smem + st * S::STAGE;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) cut4(xr[j], sp + xat[j], S::XPL);
-    cut4(gr, sp + 3 * S::XPL + gat, S::GPL);
+    for (int j = 0; j < 2; ++j) cut4(j, xr[j], sp + xat[j], S::XPL);
+    cut4(2, gr, sp + 3 * S::XPL + gat, S::GPL);
   };
   load(nx, xr, gr);
   stash(0);
@@ -3469,20 +3483,22 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
       cs.h = 0;
       if (++cs.j == cs.cnt) break;
     }
-    // (mx also covers the next task's first step, stored already: at worst the task before
+    // (range also covers the next task's first step, stored already: at worst the task before
     // one that has to be is computed twice)
-    if (mx > kBf16Max) *flag = 1;
+    if (range.outside(kTop)) *flag = 1;
     stage_barrier<63>();
+    float unscale = gdiv;
     if (__builtin_expect(*flag != 0, 0)) {
       redo(cs);
+      unscale = 1.f;
       __syncthreads();                  // every wave has read the flag
       if (threadIdx.x == 0) *flag = 0;  // (set again a whole task of barriers from here at the earliest)
     }
-    mx = 0.f;  // the next task's, from its first step (still in registers)
-    max4(xr[0]);
-    max4(xr[1]);
-    max4(gr);
-    epilogue(cs);
+    range = CutRange<3>();  // the next task's, from its first step (still in registers)
+    see4(0, xr[0]);
+    see4(1, xr[1]);
+    see4(2, gr);
+    epilogue(cs, unscale);
     if (!seek(cs.q + 1, cs)) break;
   }
 }
@@ -3714,8 +3730,8 @@ static hipError_t backward_typed(const BwdArgs& a, hipStream_t s, hipEvent_t pas
   for (int chunk = 0; chunk < (int)P.n_chunks; ++chunk) {
     const int vlo = chunk * (int)P.chunk_nvt;
     const int nv = (int)(P.nvt - vlo < P.chunk_nvt ? P.nvt - vlo : P.chunk_nvt);
-    // chunk 0 also copies the rows into the sorted order (extra workgroups)
-    const unsigned cg = 1 + (chunk == 0 && sorted_ok ? (unsigned)((a.N + 15) / 16) : 0u);
+    // chunk 0 also copies the rows into the sorted order and finds the G tiles' scale (extra workgroups)
+    const unsigned cg = 1 + (chunk == 0 && sorted_ok ? (unsigned)((a.N + 15) / 16) : 0u) + (chunk == 0 && a.g_scaled ? 1u : 0u);
     hipLaunchKernelGGL(bwd_compact_kernel, dim3(cg), dim3(1024), 0, s, a, chunk);
     if ((err = hipGetLastError()) != hipSuccess) return err;
     if (!(want_de || want_dc || want_db)) continue;

@@ -110,9 +110,10 @@ constexpr int kDcBlkChunk = 4;                         // one-tile owners per dC
 constexpr int64_t kPermMaxN = 65536;   // rows the sort handles
 constexpr int64_t kPermMaxKey = 16384; // tiles + 1 (the key of rows without gradient)
 constexpr int kPermFlag = 15;          // counts[kPermFlag]: 1 when the backward runs on sorted rows
-// counts[kGScaleExp]: fp16 G tiles hold G * 2^s with s = counts[kGScaleExp] (written by
-// the compaction from max |d_nll|, so that G's largest values sit near 2^14 and its
-// small ones stay clear of fp16's subnormal range); the sums scale back by 2^-s.
+// counts[kGScaleExp]: fp16 and fp32 G tiles hold G * 2^s with s = counts[kGScaleExp] (written by
+// the compaction from max |d_nll|, so that G's largest values sit near 2^14, in fp32 2^51,
+// and its small ones stay clear of fp16's subnormal range, in fp32 of the magnitudes that
+// three bf16 values cannot hold); the sums scale back by 2^-s.
 constexpr int kGScaleExp = 14;
 
 // Pass table: kPassInts ints per pass of the current chunk, written by the compaction.
@@ -394,7 +395,7 @@ struct BwdArgs {
   int dc_geo;           // dC sums geometry: 0 the backward's choice (filter off: wide; on: per pass), 1 wide, 2 narrow
   int dc_zeroed;        // dC already holds zeros: only rows of vocab tiles with kept tiles are written
   int stats32;          // tile_max per 32 columns in the reference's layout [N][ceil(V/32)] (else [nvt][N])
-  int g_scaled;         // fp16: G tiles hold G * 2^counts[kGScaleExp] (else unscaled)
+  int g_scaled;         // fp16, fp32: G tiles hold G * 2^counts[kGScaleExp] (else unscaled)
   int g_split;          // 16-bit: G tiles hold the hi / lo pair (else G rounded once)
   int dc_blk;           // the narrow dC sums run owners with one kept tile as tasks per (token block, D slice)
   int g_tiles_ok;       // the compaction may list G tasks by vocabulary tile, or by pair

@@ -223,6 +223,46 @@ def test_fp32_infinite_operands(m, cuda, N, D, V, filter_eps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-34, 1e-36, 1e34])
+@pytest.mark.parametrize("N,D,V", [(3, 4, 5), (257, 68, 513), (700, 512, 9000)])
+def test_fp32_products_of_tiny_values(m, cuda, N, D, V, scale):
+    """Operands below 2^-110 (e or c), which three bf16 values do not hold: the logits are as close to
+    float64 as fp32 sums (each of the D products and sums rounds by 2^-24; 2e-6 is far above their
+    2-norm).  e stays above 2^-126, where fp32 itself has no fewer bits."""
+    e, c, t = _case(N, D, V, torch.float32, cuda, seed=D, std=1.0)
+    e = torch.where(e.abs() < 0.05, torch.full_like(e, 0.05), e) * scale
+    c = torch.where(c.abs() < 0.05, torch.full_like(c, 0.05), c) / scale
+    tm, _, _, lse, _ = m._ext.forward(e, c, t)
+    x = e.double() @ c.double().T
+    want = torch.nn.functional.pad(x, (0, -V % 128), value=-float("inf")).view(N, -1, 128).amax(2).T
+    assert (tm.double() - want).norm() <= 2e-6 * want.norm()
+    assert (lse.double() - torch.logsumexp(x, 1)).norm() <= 2e-6 * torch.logsumexp(x, 1).norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cot,es,cs", [(1e-33, 1, 1), (1e-36, 1, 1), (1e30, 1, 1), (1, 1e-35, 1e34), (1, 1e34, 1e-35), (1e25, 1e-10, 1)])
+@pytest.mark.parametrize("N,D,V,eps", [(5, 4, 100, None), (5, 4, 100, -8.3177661667), (384, 260, 2000, None),
+                                       (384, 260, 2000, -8.3177661667), (130, 64, 40000, None)])
+def test_fp32_gradients_of_tiny_values(m, cuda, N, D, V, cot, es, cs, eps):
+    """fp32 gradients with cotangents, or classifier or hidden rows, whose magnitudes three bf16 values
+    do not hold, or larger than the sums' scaled range: against float64 as at ordinary magnitudes (2e-6,
+    and half of fp32's last subnormal bit for each value).  With the filter on, logits near zero and
+    V < 4096 keep every tile."""
+    e, c, t = _case(N, D, V, torch.float32, cuda, seed=N + D, std=0.02)
+    e, c = e * es, c * cs
+    t[::8] = -100
+    tm, _, _, lse, _ = m._ext.forward(e, c, t)
+    d = torch.linspace(0.5, 1.5, N, device=cuda) * cot
+    dE, dC, _ = m._ext.backward(e, c, t, lse, tm, d, filter_eps=eps)
+    G = torch.softmax(e.double() @ c.double().T, 1)
+    rows = t >= 0
+    G[rows.nonzero().flatten(), t[rows]] -= 1
+    G *= (d.double() * rows).unsqueeze(1)
+    for g, w in ((dE, G @ c.double()), (dC, G.T @ e.double())):
+        assert (g.double() - w).norm() <= 2e-6 * w.norm() + 2.0 ** -150 * w.numel() ** 0.5
+
+
+@pytest.mark.gpu
 def test_fp32_infinite_operand_stays_with_its_tasks(m, cuda):
     """An infinite classifier entry has the dE tasks of its 256 columns computed on the fp32 path, and not
     later tasks of the same workgroup: 600 tasks on 256 workgroups here, where a third of them take a
