@@ -223,6 +223,19 @@ def test_fp32_infinite_operands(m, cuda, N, D, V, filter_eps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,V", [(512, 1), (4096, 1), (4096, 300), (4100, 1)])
+def test_fp32_logits_do_not_lean(m, cuda, D, V):
+    """The mean error of 16384 fp32 logits per column: bf16 MFMA sums lean towards -inf (3e-7 of the rms logit
+    at D = 4096 as they are), which moves every lse the same way.  The random errors' mean is
+    1e-6 / 128; a third of the lean is allowed."""
+    e, c, t = _case(16384, D, V, torch.float32, cuda, seed=D, std=1.0)
+    tm, _, _, lse, _ = m._ext.forward(e, c, t)
+    x = e.double() @ c.double().T
+    want = torch.nn.functional.pad(x, (0, -V % 128), value=-float("inf")).view(16384, -1, 128).amax(2).T
+    assert abs(float((tm.double() - want).mean())) <= 1e-7 * float(x.pow(2).mean().sqrt())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("scale", [1e-34, 1e-36, 1e34])
 @pytest.mark.parametrize("N,D,V", [(3, 4, 5), (257, 68, 513), (700, 512, 9000)])
 def test_fp32_products_of_tiny_values(m, cuda, N, D, V, scale):
