@@ -1348,10 +1348,11 @@ __host__ __device__ inline int dc_bins(int nwg, int nds) {
 // dealing order.  Run by one workgroup of NT threads (the bisection by wave 0);
 // smem holds its tables.
 constexpr int kDcOwnerCost = 3;  // a task's epilogue and restart, in pipeline steps (measured at c3)
-// pipeline steps of the narrow dC sums per kept tile: one per 128-byte G row slice
+// pipeline steps of the narrow dC sums per kept tile: one per 128-byte G row slice; of the fp32
+// sums: one per 16 rows
 template <typename T>
 constexpr int dc_steps_per_tile(bool split) {
-  return kBwdVocab / (split ? 32 : 128 / (int)sizeof(T));
+  return kBwdVocab / (sizeof(T) == 4 ? 16 : split ? 32 : 64);
 }
 
 __device__ __forceinline__ int wave_min(int v) {
@@ -3180,6 +3181,7 @@ static_assert(SumCut::DN == kDcSliceCols && SumCut::DN == kDePartCols, "the task
 template <int PHASE>
 __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, int chunk, int pass, int list) {
   using S = SumCut;
+  static_assert(S::SPT == dc_steps_per_tile<float>(false), "the dC schedule counts these steps per kept tile");
   __shared__ __attribute__((aligned(16))) char smem[2 * S::STAGE + 16];
   int* const flag = reinterpret_cast<int*>(smem + 2 * S::STAGE);  // an infinity was met
   const int nrb = (int)a.plan.nrb, nds = (int)((a.D + S::DN - 1) / S::DN);
