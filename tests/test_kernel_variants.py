@@ -223,6 +223,59 @@ def test_fp32_infinite_operands(m, cuda, N, D, V, filter_eps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,D,V", [(40, 16, 300), (300, 36, 701), (600, 512, 704)])
+def test_fp32_infinite_hidden_row(m, cuda, N, D, V):
+    """An infinite entry in an ignored row of e: the forward tiles that hold it are computed again, the bias
+    included (in LDS or, for V not a multiple of 4, from memory); every other row's loss is float64's
+    (1e-5: fp32 sums) and the row itself is masked."""
+    e, c, t = _case(N, D, V, torch.float32, cuda, seed=5, std=0.5)
+    b = torch.randn(V, device=cuda)
+    e[3, 1] = float("inf")
+    t[3] = -100
+    nll = m._ext.forward(e, c, t, b)[4]
+    keep = torch.arange(N, device=cuda) != 3
+    want = torch.nn.functional.cross_entropy(e[keep].double() @ c.double().T + b.double(), t[keep], reduction="none")
+    assert nll[3] == 0 and ((nll[keep].double() - want).abs() <= 1e-5 * want.abs().clamp(min=1)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("g_tasks", [None, "blocks"])
+@pytest.mark.parametrize("what", ["infinite", "tiny"])
+@pytest.mark.parametrize("N,D,V", [(40, 16, 300), (2100, 36, 3999), (2300, 64, 4000)])
+def test_fp32_gradients_beside_the_cut(m, cuda, N, D, V, what, g_tasks):
+    """Filtered gradients of all three operands where G tiles and dC / dE tasks are computed on the fp32 path, in
+    the G kernel's pair tasks (the first size) and its tasks of up to 4 vocabulary tiles or token blocks
+    (over 512 kept pairs, last blocks partial): against float64 (2e-6, logits near zero and V < 4096
+    keep every tile).  An infinite classifier entry makes its column's logits -inf; dE's own column
+    of it holds 0 * inf and is left out."""
+    e, c, t = _case(N, D, V, torch.float32, cuda, seed=N, std=0.02)
+    b = torch.randn(V, device=cuda) * 0.01
+    keep = torch.ones(V, dtype=torch.bool, device=cuda)
+    if what == "infinite":
+        e[:, 0] = e[:, 0].abs() + 0.5
+        c[7, 0] = -float("inf")
+        keep[7] = False
+        t[t == 7] = 8
+    else:
+        e, c = e * 1e-35, c * 1e34
+    t[::8] = -100
+    tm, _, _, lse, _ = m._ext.forward(e, c, t, b)
+    d = torch.linspace(0.5, 1.5, N, device=cuda)
+    kept = torch.empty(3, dtype=torch.int64, device=cuda)
+    with m._ext.backward_options(g_tasks=g_tasks, token_order="input"):  # (sorted, the ignored rows leave blocks empty)
+        dE, dC, dB = m._ext.backward(e, c, t, lse, tm, d, b, tile_stats=kept)
+    assert kept[0] == kept[1] and (kept[0] > 512) == (N > 2000)
+    G = torch.zeros((N, V), dtype=torch.float64, device=cuda)
+    G[:, keep] = torch.softmax(e.double() @ c[keep].double().T + b[keep].double(), 1)
+    rows = t >= 0
+    G[rows.nonzero().flatten(), t[rows]] -= 1
+    G *= (d.double() * rows).unsqueeze(1)
+    skip = 1 if what == "infinite" else 0
+    for g, w in ((dE[:, skip:], G[:, keep] @ c[keep, skip:].double()), (dC, G.T @ e.double()), (dB, G.sum(0))):
+        assert (g.double() - w).norm() <= 2e-6 * w.norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,V", [(512, 1), (4096, 1), (4096, 300), (4100, 1)])
 def test_fp32_logits_do_not_lean(m, cuda, D, V):
     """The mean error of 16384 fp32 logits per column: bf16 MFMA sums lean towards -inf (3e-7 of the rms logit
@@ -403,7 +456,8 @@ def test_fp32_sums_on_bf16_mfma(m, cuda, N, D, V, eps, dc):
     rows = t >= 0
     G[rows.nonzero().flatten(), t[rows]] -= 1
     G *= (d.double() * rows).unsqueeze(1)
-    assert kept[0] == kept[1] or not rows.view(-1).any() or N % 128 == 1
+    blocks = torch.nn.functional.pad(rows, (0, -N % 128)).view(-1, 128).any(1)
+    assert kept[0] == blocks.sum() * ((V + 127) // 128)
     for g, w in ((dE, G @ c.double()), (dC, G.T @ e.double())):
         assert (g.double() - w).norm() <= 2e-6 * w.norm()
 
