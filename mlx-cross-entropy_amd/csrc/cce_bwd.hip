@@ -608,11 +608,13 @@ struct RowData {
   const float* lse;
   const float* d_nll;
   const int* map;
+  int gexp;  // the G tiles hold G 2^gexp (fp16 and fp32; 0 unless a.g_scaled)
 };
 __device__ __forceinline__ RowData row_data(const BwdArgs& a) {
+  const int gexp = a.g_scaled ? ldu(a.counts, kGScaleExp) : 0;
   if (a.perm && ldu(a.counts, kPermFlag) != 0)
-    return RowData{reinterpret_cast<const char*>(a.e_perm), a.t_perm, a.lse_perm, a.dnll_perm, a.perm};
-  return RowData{reinterpret_cast<const char*>(a.e), a.targets, a.lse, a.d_nll, nullptr};
+    return RowData{reinterpret_cast<const char*>(a.e_perm), a.t_perm, a.lse_perm, a.dnll_perm, a.perm, gexp};
+  return RowData{reinterpret_cast<const char*>(a.e), a.targets, a.lse, a.d_nll, nullptr, gexp};
 }
 
 // Row copy into the sorted order, when the compaction chose it: one wave per row,
@@ -1531,9 +1533,6 @@ __device__ __forceinline__ GRows g_rows_load(const BwdArgs& a, const RowData& rd
   return r;
 }
 
-// The exponent s of the fp16 and fp32 G tiles' scale 2^s (0 unless a.g_scaled).
-__device__ __forceinline__ int g_scale_exp(const BwdArgs& a) { return a.g_scaled ? ldu(a.counts, kGScaleExp) : 0; }
-
 template <typename T, bool HAS_BIAS, bool WANT_G, bool WANT_DB, int TI = 4>
 __device__ __forceinline__ void g_block_epilogue(const BwdArgs& a, const RowData& rd, const f32x16 (&w)[TI][2],
                                                  int64_t v0, int64_t tok0, int row0, char* gtile, float* red,
@@ -1544,8 +1543,7 @@ __device__ __forceinline__ void g_block_epilogue(const BwdArgs& a, const RowData
   const T* bias = reinterpret_cast<const T*>(a.bias);
   // fp16, fp32: G is formed as (d_nll 2^s) (p - onehot), exact scaling by a power of two;
   // the column sums take it back out
-  const int gexp = g_scale_exp(a);
-  const float gmul = __builtin_ldexpf(1.f, gexp), gdiv = __builtin_ldexpf(1.f, -gexp);
+  const float gmul = __builtin_ldexpf(1.f, rd.gexp), gdiv = __builtin_ldexpf(1.f, -rd.gexp);
   float g[TJ], lz[TJ];
   int tl[TJ];
   GRows gr;
@@ -2484,7 +2482,7 @@ __global__ __launch_bounds__((SumGeo<T, SPLIT>::NT), 1) void bwd_sum_kernel(BwdA
   constexpr int RK = 8 + (PHASE == 0 ? 2 : 4);
   constexpr int MK = 8;
   // fp16 G tiles hold G 2^gexp: the epilogue scales the sums back (exact)
-  const float gdiv = __builtin_ldexpf(1.f, -g_scale_exp(a));
+  const float gdiv = __builtin_ldexpf(1.f, -rd.gexp);
 
   // acc[i][jj][r]: output column ds DN + 128 wd + 32 i + 8 (r/4) + 4 h + r%4 of row 64 wm + 32 jj + n.
   auto epilogue = [&](const Cur& c) {
@@ -2890,7 +2888,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_sum_narrow_kernel(BwdArgs a, 
         for (int jj = 0; jj < 2; ++jj) acc[i][jj] = Traits<T>::mfma(x[i], g[hl][jj], acc[i][jj]);
   };
   // fp16 G tiles hold G 2^gexp: the epilogue scales the sums back (exact)
-  const float gdiv = __builtin_ldexpf(1.f, -g_scale_exp(a));
+  const float gdiv = __builtin_ldexpf(1.f, -rd.gexp);
 
   // acc[i][jj][r]: output column ds DN + 128 wd + 32 i + 8 (r/4) + 4 h + r%4 of row 64 wm + 32 jj + n.
   auto epilogue = [&](const Cur& c) {
@@ -3342,7 +3340,7 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
   };
 
   f32x16 acc[2][2];
-  const float gdiv = __builtin_ldexpf(1.f, -g_scale_exp(a));  // G tiles hold G 2^gexp: scaled back (exact)
+  const float gdiv = __builtin_ldexpf(1.f, -rd.gexp);  // G tiles hold G 2^gexp: scaled back (exact)
   // The task once more on fp32 MFMAs, fragments from memory, G unscaled.
   auto redo = [&](Cur c) {
 #pragma unroll
