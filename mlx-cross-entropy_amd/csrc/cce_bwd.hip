@@ -1572,14 +1572,19 @@ __device__ __forceinline__ void g_block_epilogue(const BwdArgs& a, const RowData
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int c = i * 32 + (r >> 2) * 8 + (r & 3);
+      // fp32: the logit as the forward rounds it (the sum, then the bias), so that its rounding
+      // cancels against lse's in confident rows; with the bias in the exponent's constant, a class'
+      // rounding there is the same for all its tokens, and adds up in dC
+      constexpr bool LOGIT = ES == 4;
       float add = 0.f;
       if (HAS_BIAS) {
         const int64_t v = v0 + c + 4 * h;
-        add = v < a.V ? to_f32(bias[v]) * kLog2e : 0.f;
+        add = v < a.V ? to_f32(bias[v]) * (LOGIT ? 1.f : kLog2e) : 0.f;
       }
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(w[i][j][r], kLog2e, add - lz[j]));
+        const float p = LOGIT ? __builtin_amdgcn_exp2f(fmaf(HAS_BIAS ? w[i][j][r] + add : w[i][j][r], kLog2e, -lz[j]))
+                              : __builtin_amdgcn_exp2f(fmaf(w[i][j][r], kLog2e, add - lz[j]));
         gv[j][r] = g[j] * p - (tl[j] == c ? g[j] : 0.f);
       }
     }

@@ -83,10 +83,10 @@ __device__ __forceinline__ void fwd_store_pending(const FwdArgs& a, const FwdPen
 }
 
 // How a tile kernel adds the bias: none; from global memory after the contraction
-// (fwd_add_bias); or as the accumulators' starting value, staged through LDS
-// (fwd_stage_bias / fwd_init_bias_lds), when the bias is 16-byte aligned and
-// V * sizeof(T) is a multiple of 16 (no 16-byte piece of the bias then straddles its
-// end).  The two orders of the fp32 sums differ in the last bits.
+// (fwd_add_bias); or staged through LDS (fwd_stage_bias / fwd_bias_from_lds), when the
+// bias is 16-byte aligned and V * sizeof(T) is a multiple of 16 (no 16-byte piece of the
+// bias then straddles its end): as the accumulators' starting value (16-bit types; the two
+// orders of the sums differ in the last bits), or after the contraction (fp32; kBiasFirst).
 enum FwdBias { kBiasNone = 0, kBiasGlobal = 1, kBiasLds = 2 };
 
 // The bias of the wave's 128 vocabulary rows added to a tile's logits.  The tile
@@ -114,8 +114,8 @@ __device__ __forceinline__ void fwd_add_bias(const FwdArgs& a, f32x16 (&acc)[TI]
 // The bias through LDS (kBiasLds).  Per tile the block's kFwdVocab bias values (1
 // KiB at most; zeros past V) are copied into an LDS buffer by one LDS-DMA load of
 // wave 0, issued ahead of the tile's pipeline fill, so that the tile's first stage
-// barrier, which waits for all of a wave's loads, covers it.  Right after that barrier
-// the accumulators are set to the bias (fwd_init_bias_lds), and the MFMAs add the
+// barrier, which waits for all of a wave's loads, covers it.  In 16 bits, right after that barrier
+// the accumulators are set to the bias (fwd_bias_from_lds), and the MFMAs add the
 // products to it: no bias work is left in the epilogue, where 64 global loads per
 // lane cost 7% of the forward at N = 4096, D = 2304, V = 256000 (adding from LDS
 // there still 4%: the added registers spilled).  The buffer is rewritten at the end
@@ -140,9 +140,18 @@ __device__ __forceinline__ void fwd_stage_bias(const FwdArgs& a, int vb, char* b
                                                   : reinterpret_cast<const char*>(g_zero16);
   dma16(g, __builtin_amdgcn_readfirstlane(lds_addr(buf)));
 }
-// acc[i][j][r] = the bias of the register's vocabulary column (see fwd_epilogue's layout).
-template <typename T, int TI, int TJ>
-__device__ __forceinline__ void fwd_init_bias_lds(const char* buf, f32x16 (&acc)[TI][TJ]) {
+// fp32 adds it after the contraction instead: the dense G kernel forms the same product without
+// a bias, and where the two are the same bits, the bias added the same way, a logit's
+// rounding cancels against lse's in softmax - 1 of a confident row.  Started from the bias, the sums round
+// elsewhere: dE of peaked rows at N = 700, D = 4096, V = 1000 was then off by 1.6e-5 of float64, now
+// 6.1e-6, dC 1.5e-5 and 5.3e-6 (fp32 MFMAs, started from the bias: 2.1e-5 and 1.9e-5).  The forward at N =
+// 1000, D = 1024, V = 50000 takes 579 -> 588 us for it.
+template <typename T>
+constexpr bool kBiasFirst = sizeof(T) == 2;
+
+// acc[i][j][r] = (ADD: +=) the bias of the register's vocabulary column (see fwd_epilogue's layout).
+template <typename T, bool ADD, int TI, int TJ>
+__device__ __forceinline__ void fwd_bias_from_lds(const char* buf, f32x16 (&acc)[TI][TJ]) {
   const int lane = lane_here();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c0 = (wave & 1) * 128 + (lane >> 5) * 4;
@@ -166,7 +175,7 @@ __device__ __forceinline__ void fwd_init_bias_lds(const char* buf, f32x16 (&acc)
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j][4 * q + k] = add[k];
+        for (int j = 0; j < TJ; ++j) acc[i][j][4 * q + k] = ADD ? acc[i][j][4 * q + k] + add[k] : add[k];
     }
   }
 }
@@ -349,19 +358,19 @@ __global__ __launch_bounds__(FwdLoop<T>::NTHREADS, 1) void fwd_tile_kernel(FwdAr
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool active = (int64_t)tb * kFwdTokens + (wave >> 1) * (kFwdTokens / kFwdWB) < a.N &&
                         (int64_t)vb * kFwdVocab + (wave & 1) * 128 < a.V;
-    // kBiasLds: the accumulators start from the tile's bias (in LDS after the first stage barrier)
+    // kBiasLds: 16-bit accumulators start from the tile's bias (in LDS after the first stage barrier)
     if constexpr (S32) {
       Loop::template consume<RAGGED>(
           src, smem, acc,
           [&]() {
-            if constexpr (BIAS == kBiasLds) fwd_init_bias_lds<T>(bias_lds, acc);
+            if constexpr (BIAS == kBiasLds && kBiasFirst<T>) fwd_bias_from_lds<T, false>(bias_lds, acc);
           },
           false, active);
     } else {
       Loop::template consume<RAGGED>(
           src, smem, acc,
           [&]() {
-            if constexpr (BIAS == kBiasLds) fwd_init_bias_lds<T>(bias_lds, acc);
+            if constexpr (BIAS == kBiasLds && kBiasFirst<T>) fwd_bias_from_lds<T, false>(bias_lds, acc);
             fwd_store_pending(a, pend, ptb, pvb);
           },
           false, active);
@@ -374,6 +383,10 @@ __global__ __launch_bounds__(FwdLoop<T>::NTHREADS, 1) void fwd_tile_kernel(FwdAr
     const int tbn = walk.tb, vbn = walk.vb;
     int64_t tgn[TJ];
     if constexpr (BIAS == kBiasGlobal) fwd_add_bias<T>(a, acc, vb);
+    if constexpr (BIAS == kBiasLds && !kBiasFirst<T>) {
+      fwd_bias_from_lds<T, true>(bias_lds, acc);
+      if (more) __syncthreads();  // every wave has read the buffer
+    }
     if (more) {
       if constexpr (BIAS == kBiasLds) fwd_stage_bias<T>(a, vbn, bias_lds);
       src = sources(tbn, vbn);

@@ -276,6 +276,29 @@ def test_fp32_gradients_beside_the_cut(m, cuda, N, D, V, what, g_tasks):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,D,V", [(300, 512, 1000), (700, 4096, 1000), (700, 4096, 1002), (2500, 2048, 5000)])
+def test_fp32_confident_rows_with_a_bias(m, cuda, N, D, V):
+    """softmax - 1 of confident rows is what is left of exp(logit - lse): the logit's own rounding cancels
+    when the dense G kernel forms the bits the forward formed, the bias included (in LDS or from
+    memory).  What stays is the rounding of lse and of its product with log2(e), half an ulp each: the
+    error of G at the target, from dE along c_t, is below 2^-24 of lse (2-norm over the rows)."""
+    g = torch.Generator(device=cuda).manual_seed(D)
+    c = torch.randn((V, D), generator=g, device=cuda) * 0.02
+    b = torch.randn(V, generator=g, device=cuda) * 0.1
+    t = torch.randint(0, V, (N,), generator=g, device=cuda)
+    ct = c[t]
+    e = ct * (14 / ct.pow(2).sum(1, keepdim=True)) + 0.5 * torch.randn((N, D), generator=g, device=cuda)
+    tm, _, _, lse, _ = m._ext.forward(e, c, t, b)
+    dE = m._ext.backward(e, c, t, lse, tm, torch.ones(N, device=cuda), b, filter_eps=None, want_dc=False)[0]
+    x = e.double() @ c.double().T + b.double()
+    l = torch.logsumexp(x, 1)
+    G = torch.exp(x - l.unsqueeze(1))
+    G[torch.arange(N, device=cuda), t] -= 1
+    err = ((dE.double() - G @ c.double()) * ct.double()).sum(1) / ct.double().pow(2).sum(1)
+    assert err.pow(2).mean().sqrt() <= 2.0 ** -24 * l.mean()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,V", [(512, 1), (4096, 1), (4096, 300), (4100, 1)])
 def test_fp32_logits_do_not_lean(m, cuda, D, V):
     """The mean error of 16384 fp32 logits per column: bf16 MFMA sums lean towards -inf (3e-7 of the rms logit
