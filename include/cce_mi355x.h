@@ -200,6 +200,9 @@ int cce_backward(int dtype, const void* e, const void* c, const void* bias,
  * results agree to rounding either way): */
 #define CCE_BWD_TOKENS_INPUT 2    /* token blocks of 128 rows in input order */
 #define CCE_BWD_TOKENS_SORTED 4   /* token blocks of the rows grouped by target tile, when available */
+/* 16-bit inputs: the sums' tasks.  fp32 inputs have 256-column tasks only: the DE flags are
+ * ignored, the DC ones choose how owners are dealt to workgroups (WIDE in turn, as dE's; NARROW
+ * longest first) and, with the filter off, the G kernel, as for 16-bit inputs. */
 #define CCE_BWD_DE_SUMS_WIDE 8    /* dE sums in 512-column tasks */
 #define CCE_BWD_DE_SUMS_NARROW 16 /* dE sums in 256-column tasks */
 #define CCE_BWD_DC_SUMS_WIDE 32   /* dC sums in 512-column tasks */
@@ -210,8 +213,9 @@ int cce_backward(int dtype, const void* e, const void* c, const void* bias,
 /* Launch the passes of the dense worst case and let the device skip the ones the data
  * does not need, instead of waiting on the host, once per vocabulary chunk, for the
  * compaction's pass count (which then launches exactly the passes needed).  The wait
- * is skipped anyway while the stream is being captured into a graph, and by
- * cce_backward_noalloc. */
+ * is skipped anyway while the stream is being captured into a graph, by
+ * cce_backward_noalloc, and when the sizes leave one chunk and one pass whatever the data
+ * (only the dC geometry is then left open: both are launched). */
 #define CCE_BWD_DEVICE_PASSES 256
 /* Precision of the softmax gradient G between the backward's two products (16-bit
  * inputs; fp32 inputs keep G in fp32).  By default G is carried as a pair of 16-bit
@@ -229,8 +233,9 @@ int cce_backward(int dtype, const void* e, const void* c, const void* bias,
 /* With the filter on and the kept tiles shared by three or more token blocks on
  * average, the G kernel's tasks are a vocabulary tile with up to 4 of its kept blocks
  * (the tile's C rows read once for them), not a token block with up to 4 of its kept
- * tiles.  This keeps the token-block tasks (the G values can differ in the last bits:
- * the contraction's slices are summed in another order). */
+ * tiles.  With at most two kept pairs per workgroup a task is one pair, spread over the whole
+ * workgroup.  This keeps the token-block tasks in both cases (the G values can differ in the
+ * last bits: the contraction's slices are summed in another order). */
 #define CCE_BWD_G_TASKS_BY_BLOCK 4096
 /* When a pass has at most half as many (128-row block, 256-column D slice) dE tasks
  * as workgroups (small N and D), each task is cut along its kept tiles into pieces

@@ -3165,11 +3165,12 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_sum_narrow_kernel(BwdArgs a, 
 // and columns past D read zeros), are cut there and stored to LDS while the step before is
 // multiplied.  X, and G for dC, are planes of natural rows read transposed; G for dE is in
 // the NT loop's fragment order.  With `list` the dC tasks are dealt like dE's (snake order over
-// own_vt: the filter off, or evenly shared tiles), else by the schedule's bins.  MFMA-bound,
-// LDS reads next (half of the MFMAs' time).  At N = 1000, D = 1024, V = 50000, all tiles
-// kept: dE 608 us, dC 718 us; the fp32 MFMA kernels before took 846 and 1025 (N = 512, D = 512,
-// V = 32000, filtered: 37 and 42 us, before 52 and 55).  dE and dC are closer to float64 than
-// with fp32 MFMAs (8.8e-7 against 1.4e-6 in the first case).
+// own_vt: the filter off, or evenly shared tiles), else by the schedule's bins.  Bound by the
+// MFMAs (the matrix pipe busy 40 to 46% of the SIMD cycles) and the cut, LDS reads (half of the MFMAs'
+// time) and barriers beside them.  At N = 1000, D = 1024, V = 50000, all tiles kept: dE 600 us, dC 680
+// us; the fp32 MFMA kernels before took 846 and 1025 (N = 512, D = 512, V = 32000, filtered: 38 and 42
+// us, before 52 and 55).  dE and dC are closer to float64 than with fp32 MFMAs (8.8e-7 against 1.4e-6
+// in the first case).
 struct SumCut {
   static constexpr int NT = 512, DN = 256, KS = 16;
   static constexpr int SPT = kBwdVocab / KS;      // steps per kept tile
@@ -3669,8 +3670,9 @@ static void launch_sum(const BwdArgs& a, bool wide, int chunk, int pass, int gri
 // rounds of equal tasks over the persistent grid.  With the filter on the owners' kept
 // counts differ, and two or four wide tasks per workgroup balance worse than twice as
 // many narrow ones (c3: the wide tasks' 18 to 28 kept tiles per workgroup; narrow
-// measured 10-13 us faster at c3 and c4), so the filter on takes the narrow one.
-// a.de_geo forces one (1 wide, 2 narrow).
+// measured 10-13 us faster at c3 and c4), so the filter on takes the narrow one.  (Not a line
+// between the two: with 16 wide tasks per workgroup, N = 32768, D = 8192, the wide one takes
+// 0.7 ms less of a 67 ms step.)  a.de_geo forces one (1 wide, 2 narrow).
 static bool use_wide_de_sums(const BwdArgs& a, int grid) {
   if (a.plan.esize == 4) return false;  // fp32 has one geometry
   if (a.de_geo != 0) return a.de_geo == 1;

@@ -105,7 +105,7 @@ def backward_options(token_order=None, de_sums=None, dc_sums=None, max_g_tiles=0
     with the filter off and a single rounding with it on); dc_tasks "owners" (the
     narrow dC sums run one-tile owners as owner tasks, not grouped by token block);
     g_tasks "blocks" (the G kernel's tasks are token blocks with up to 4 kept tiles,
-    never vocabulary tiles with up to 4 kept blocks); de_tasks "whole" (the dE sums never
+    never vocabulary tiles with up to 4 kept blocks, nor single pairs); de_tasks "whole" (the dE sums never
     cut a (token block, D slice) task into pieces); dc_zero_fill "forward" (the
     autograd op has the forward's tile kernel zero dC, cce_forward_ex, and the backward
     write only the rows of kept tiles, CCE_BWD_DC_ZEROED) | "backward" (the default:
@@ -555,7 +555,8 @@ QUANT_SCRATCH_BYTES = 512 << 20  # dequantized rows at a time (the G tiles' budg
 
 def quant_chunk_rows(qw):
     """Rows the autograd op dequantizes at a time: as many as QUANT_SCRATCH_BYTES hold (a
-    multiple of 4096), at least the library's default of 32768.  Every chunk costs a
+    multiple of 4096), at least the library's default of 32768; all of them, in scratch, when
+    the dequantized matrix is smaller than that.  Every chunk costs a
     dequantization and a tile launch forward, and a compaction, a G kernel and sums backward,
     each at least a task long however few its rows.  Steps in us with 32768 rows / 256 MiB /
     512 MiB / 1 GiB a chunk: 4 bits, N = 2000, D = 4096, V = 128256 2783 / 2776 / 2550 / 2304

@@ -13,7 +13,10 @@ Here the quantized rows go to the loss as they are:
     loss = linear_cross_entropy(hidden, qw, targets)
 
 and the HIP library dequantizes a bounded chunk of rows at a time (cce_forward_q /
-cce_backward_q) instead of materialising the [V, D] matrix.  The rows carry no
+cce_backward_q).  The loss takes chunks of up to 512 MiB of dequantized rows
+(_ext.quant_chunk_rows), so that a larger [V, D] matrix is never materialised whole, and a
+smaller one is, in scratch, for the length of the call; forward_q / backward_q take any
+chunk_rows.  The rows carry no
 gradient (the frozen-head setting of those callers); dE and dBias are produced.
 
 Layout (MLX's, mlx >= 0.22): ``weight`` [V, D * bits / 32] 32-bit words, code j of a
