@@ -215,7 +215,7 @@ int cce_backward(int dtype, const void* e, const void* c, const void* bias,
  * compaction's pass count (which then launches exactly the passes needed).  The wait
  * is skipped anyway while the stream is being captured into a graph, by
  * cce_backward_noalloc, and when the sizes leave one chunk and one pass whatever the data
- * (only the dC geometry is then left open: both are launched). */
+ * (only the dC geometry is then left open: for 16-bit inputs both are launched). */
 #define CCE_BWD_DEVICE_PASSES 256
 /* Precision of the softmax gradient G between the backward's two products (16-bit
  * inputs; fp32 inputs keep G in fp32).  By default G is carried as a pair of 16-bit

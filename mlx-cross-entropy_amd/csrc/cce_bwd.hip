@@ -3164,8 +3164,9 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_sum_narrow_kernel(BwdArgs a, 
 // (dC) values of G go from memory into registers (buffer loads: rows past the operand's end
 // and columns past D read zeros), are cut there and stored to LDS while the step before is
 // multiplied.  X, and G for dC, are planes of natural rows read transposed; G for dE is in
-// the NT loop's fragment order.  With `list` the dC tasks are dealt like dE's (snake order over
-// own_vt: the filter off, or evenly shared tiles), else by the schedule's bins.  Bound by the
+// the NT loop's fragment order.  With list 1 the dC tasks are dealt like dE's (snake order over
+// own_vt: the filter off, or evenly shared tiles), with 0 by the schedule's bins, with -1 as
+// the compaction picked (one launch, whether the host knows the pick or not).  Bound by the
 // MFMAs (the matrix pipe busy 40 to 46% of the SIMD cycles) and the cut, LDS reads (half of the MFMAs'
 // time) and barriers beside them.  At N = 1000, D = 1024, V = 50000, all tiles kept: dE 600 us, dC 680
 // us; the fp32 MFMA kernels before took 846 and 1025 (N = 512, D = 512, V = 32000, filtered: 38 and 42
@@ -3194,8 +3195,6 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
   const int* pi = a.pinfo + pass * kPassInts;
   const int pmode = ldu(pi, kPiDeMode);
   if (pmode < 0) return;  // past the passes the data needs
-  // the filtered backward may launch both ways of dealing dC tasks; the compaction picked one
-  if (PHASE == 1 && a.dc_geo == 0 && a.filter_log_eps > -INFINITY && ldu(pi, kPiDcWide) != list) return;
   const int s0 = ldu(pi, kPiS0);  // the G scratch holds slot s at s - s0
   const int ntasks = ldu(pi, PHASE == 0 ? kPiOwnRb : kPiOwnVt) * nds;
   int tbase = 0, ncut = 0, npc = 1;
@@ -3211,7 +3210,7 @@ __global__ __launch_bounds__(SumCut::NT, 1) void bwd_sum_cut_kernel(BwdArgs a, i
   const int dcb = dc_bins(nwg, nds);
   const int dcm = dcb > 0 ? vwg / nds : 0;
   const int ds0 = dcb > 0 ? vwg - dcm * nds : vwg;
-  const bool bins = PHASE == 1 && !list;
+  const bool bins = PHASE == 1 && (list < 0 ? ldu(pi, kPiDcWide) : list) == 0;
   const bool dc_mine = bins && (dcb > 0 ? dcm < dcb : ds0 < nds);
   const int bstart = dc_mine ? ldu(a.dc_bin_start, dcm) : 0;
   const int bcnt = dc_mine ? ldu(a.dc_bin_start, dcm + 1) - bstart : 0;
@@ -3654,7 +3653,8 @@ static void launch_sum(const BwdArgs& a, bool wide, int chunk, int pass, int gri
     }
   }
   if constexpr (sizeof(T) == 4) {
-    hipLaunchKernelGGL((bwd_sum_cut_kernel<PHASE>), dim3(grid), dim3(SumCut::NT), 0, s, a, chunk, pass, wide ? 1 : 0);
+    static_assert(PHASE == 0, "fp32 dC: launch_sums");
+    hipLaunchKernelGGL((bwd_sum_cut_kernel<PHASE>), dim3(grid), dim3(SumCut::NT), 0, s, a, chunk, pass, 1);
   } else {
     if (wide)
       hipLaunchKernelGGL((bwd_sum_kernel<T, PHASE, false>), dim3(grid), dim3(SumGeo<T, false>::NT), 0, s, a, chunk,
@@ -3687,7 +3687,7 @@ static bool use_wide_de_sums(const BwdArgs& a, int grid) {
 // geometry runs ~35% faster.  With the filter on the compaction picks one per pass
 // (kPiDcWide): narrow when one owner keeps so many blocks that its tasks outlast a
 // workgroup's average share (skewed targets, c3), else wide (c2, c4: 50-55 us faster).
-// The host then launches both kernels and the one not picked returns at once: one
+// In 16 bits the host then launches both kernels and the one not picked returns at once: one
 // kernel holding both bodies spilled the narrow one's registers (measured 50-90 us
 // slower).  This function decides the dense G kernel and the forced choices; a.dc_geo
 // forces one (1 wide, 2 narrow).
@@ -3767,7 +3767,7 @@ static hipError_t backward_typed(const BwdArgs& a, hipStream_t s, hipEvent_t pas
     };
     // The sums of one pass; dc_pick: the dC geometry the compaction chose for it (1
     // wide, 0 narrow), or -1 when unknown on the host (both are launched, and the one
-    // not chosen returns at once).
+    // not chosen returns at once; fp32 has one kernel for both).
     auto launch_sums = [&](int pass, int dc_pick) {
       hipError_t e2;
       if (want_de) {
@@ -3787,10 +3787,15 @@ static hipError_t backward_typed(const BwdArgs& a, hipStream_t s, hipEvent_t pas
         }
       }
       if (want_dc) {
-        const bool narrow = auto_dc ? dc_pick != 1 : !wide_dc;
-        const bool wide = auto_dc ? dc_pick != 0 : wide_dc;
-        if (narrow) launch_sum<T, 1>(a, false, chunk, pass, gp, s);
-        if (wide) launch_sum<T, 1>(a, true, chunk, pass, gp, s);
+        if constexpr (sizeof(T) == 4) {
+          hipLaunchKernelGGL((bwd_sum_cut_kernel<1>), dim3(gp), dim3(SumCut::NT), 0, s, a, chunk, pass,
+                             auto_dc ? -1 : wide_dc ? 1 : 0);
+        } else {
+          const bool narrow = auto_dc ? dc_pick != 1 : !wide_dc;
+          const bool wide = auto_dc ? dc_pick != 0 : wide_dc;
+          if (narrow) launch_sum<T, 1>(a, false, chunk, pass, gp, s);
+          if (wide) launch_sum<T, 1>(a, true, chunk, pass, gp, s);
+        }
         if ((e2 = hipGetLastError()) != hipSuccess) return e2;
       }
       if (want_db) {

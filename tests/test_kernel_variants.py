@@ -485,6 +485,27 @@ def test_fp32_sums_on_bf16_mfma(m, cuda, N, D, V, eps, dc):
         assert (g.double() - w).norm() <= 2e-6 * w.norm()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("skewed", [False, True])
+@pytest.mark.parametrize("passes", [None, "device"])
+@pytest.mark.parametrize("N,D,V,max_g", [(300, 260, 3000, 0), (2000, 64, 9000, 0), (2000, 64, 9000, 1)])
+def test_fp32_dc_dealt_as_picked(m, cuda, N, D, V, max_g, passes, skewed):
+    """The filtered fp32 dC sums deal their owners as the compaction picked, in one launch: the same
+    bits as with either way of dealing forced (an owner's sum does not depend on who runs it), with
+    evenly shared tiles and with most targets in one, in one pass and several."""
+    e, c, t = _case(N, D, V, torch.float32, cuda, seed=N, std=0.3)
+    if skewed:
+        t[: N * 3 // 4] = 5
+    tm, _, _, lse, _ = m._ext.forward(e, c, t)
+    d = torch.linspace(0.5, 1.5, N, device=cuda)
+    out = []
+    for dc in (None, "wide", "narrow"):
+        with m._ext.backward_options(dc_sums=dc, passes=passes, max_g_tiles=max_g):
+            out.append(m._ext.backward(e, c, t, lse, tm, d))
+    for other in out[1:]:
+        assert torch.equal(out[0][0], other[0]) and torch.equal(out[0][1], other[1])
+
+
 @pytest.mark.parametrize("V,D,dtype,rows", [
     (128256, 4096, torch.bfloat16, 65536), (128256, 4096, torch.float32, 32768), (32000, 16384, torch.bfloat16, 32768),
     (245631, 128, torch.float32, 1048576), (100000, 768, torch.bfloat16, 348160)])
